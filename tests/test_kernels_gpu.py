@@ -171,6 +171,32 @@ def test_linear_x_stationary_variant_bit_identical(hip_device, m, n, k):
            "variant 9 against the float64 reference")
 
 
+@pytest.mark.parametrize(
+    "m,n,k",
+    [(1, 32, 64), (33, 40, 64), (77, 2048, 512), (1000, 200, 128), (52, 1024, 4096), (1600, 1024, 1024),
+     (5673, 520, 192), (8191, 1000, 320), (16640, 1024, 2112)],
+)
+def test_linear_ring_tiles_bit_identical(hip_device, m, n, k):
+    """The built-in choice at K % 64 == 0 (ring kernel: tiles from 32 x 32 to 256 x 256, one to
+    many K chunks per ring, ragged M and N) accumulates the same MFMAs in the same order as the
+    pinned 64 x 128 tile: identical outputs for every epilogue, output type and the in-place residual."""
+    from tiktoktechjam2026_amd.mixed_precision.hip_linear import (
+        mixed_linear, mixed_linear_q_scaled, mixed_linear_residual)
+
+    print(f"\n[linear ring] m={m} n={n} k={k}", flush=True)
+    lin = _linear(k, n, hip_device, 61)
+    x = _randn((m, k), 67).to(hip_device, torch.float16)
+    for out_dtype in (torch.float32, torch.float16):
+        for gelu in (False, True):
+            y0, y4 = (mixed_linear(x, lin, output_dtype=out_dtype, fuse_gelu=gelu, variant=v) for v in (0, 4))
+            assert torch.equal(y0, y4), f"out={out_dtype} gelu={gelu}"
+    q0, q4 = (mixed_linear_q_scaled(x, lin, n // 16 * 8, 0.25503486, variant=v) for v in (0, 4))
+    assert torch.equal(q0, q4)
+    r = _randn((m, n), 71).to(hip_device)
+    want = mixed_linear_residual(x, lin, r, variant=4)
+    assert torch.equal(mixed_linear_residual(x, lin, r, out=r), want)
+
+
 @pytest.mark.parametrize("n,variant", [(8, 0), (256, 7), (128, 1)])
 def test_gelu_epilogue_accuracy(hip_device, n, variant):
     """The GEMM's GELU alone: X = [v, 0, ...] and W[:, 0] = 1 make every pre-activation

@@ -868,6 +868,224 @@ static hipError_t launch_linear_dma(const LinearArgs& a, hipStream_t s) {
   return launch_linear_big<256, 256, 64, 2, XT, EPI, OT>(a, s);
 }
 
+// ---- ring projection (FP16 X, K % 64 == 0): one tile per workgroup, tile chosen by the call ----
+// Calls whose 256 x 256 tiles would leave CUs idle used to run linear_kernel, which loads a
+// chunk, waits for it and multiplies it: a memory latency per 64 k values with nothing in
+// flight behind it.  Here the operands travel as in linear_dma_kernel (LDS-DMA copies, rows
+// past M / N copying the last existing row) through a ring of NS stages of 64 k values, so
+// NS - 1 chunks are in flight while one is multiplied; what bounds a small call is then the
+// K / 64 barrier steps of one tile (0.1 us each at 32 x 32), and a large one the LDS (fragment
+// reads and copies together move 1.3 x what the MFMAs of a 64 x 64 wave tile leave time for)
+// and the stores of its tile ends.
+//
+// Per chunk: read the second k-step's fragments, multiply the first's, wait for the copies of
+// the next chunk, one barrier, refill the stage just read, read the next chunk's first
+// fragments, multiply the second's.  So fragment reads run half a chunk ahead of the MFMAs that
+// use them and a barrier separates 64 k values.  The barrier follows every wave's lgkmcnt(0),
+// so no wave still reads the stage that is refilled after it.
+//
+// A staged row is 128 bytes (eight 16-byte units); unit c of row R sits in slot c ^ ((R / 2) % 8),
+// with which the 16-lane phases of a b128 fragment read cover all 64 banks once.
+// MFMAs, k order and epilogue arithmetic are those of every other variant: bit-identical results.
+//
+// Measured on MI355X, us per call, linear_kernel's best tile -> this kernel (tile):
+//   77 x 2048 x 512 GELU        13.1 -> 4.0 (32 x 32)     52 x 1024 x 4096 residual  78 -> 10.2 (32 x 64)
+//   472 x 3072 x 1024           25.3 -> 8.3 (128 x 64)    472 x 1024 x 4096 residual 165 -> 13.4 (32 x 64)
+//   1600 x 1024 x 1024          24.7 -> 8.2 (128 x 64)    5673 x 512 x 2048 residual 87 -> 23.4 (64 x 64)
+//   8192 x 1024 x 1024          41.8 -> 20.7 (128 x 128)  8192 x 8192 x 8192 (variant 8) 1206 -> 932 (256 x 256)
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NS, int EPI, typename OT>
+__global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void linear_ring_kernel(LinearArgs a) {
+  constexpr int BK = 64, ROW = BK * 2;        // bytes of a staged row
+  constexpr int NW = WAVES_M * WAVES_N;
+  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
+  constexpr int TM = WM / 16, PN = WN / 32;
+  constexpr int XBYTES = BM * ROW, SBYTES = (BM + BN) * ROW;
+  constexpr int COPIES = SBYTES / 1024, CPW = COPIES / NW;  // 1-KB copies (8 rows) per chunk: all, per wave
+  static_assert(TM * 16 == WM && PN * 32 == WN, "wave tile");
+  static_assert(CPW * NW == COPIES && NS >= 2 && (NS - 1) * CPW < 64, "copies");
+  static_assert(EPI == kEpiBias || EPI == kEpiBiasGelu || EPI == kEpiBiasResidual, "plain epilogues");
+  __shared__ __align__(16) unsigned char stages[NS * SBYTES];
+  auto swz = [](int row) { return (row >> 1) & 7; };
+
+  const _Float16* __restrict__ X = static_cast<const _Float16*>(a.x);
+  const _Float16* __restrict__ W = a.w;
+  const int64_t M = a.m;
+  const int N = a.n, K = a.k;
+  const int nbn = (N + BN - 1) / BN;
+  const int nk = K / BK;
+  const int tile = xcd_local_tile(blockIdx.x, gridDim.x);
+  const int64_t m0 = (int64_t)(tile / nbn) * BM;
+  const int n0 = (tile % nbn) * BN;
+  const int l = threadIdx.x & 63, wave = wave_id();
+  const int r = l & 15, g = l >> 4;
+  const int wm = wave % WAVES_M, wn = wave / WAVES_M;
+
+  // this wave's copies of a chunk: stage rows [0, BM) hold X, the BN after them W in w_slot order
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void*)stages;
+  const int xmax = (int)min<int64_t>(BM, M - m0) - 1, wmax = min(BN, N - n0) - 1;
+  uint32_t off[CPW];
+  const _Float16* src[CPW];
+#pragma unroll
+  for (int j = 0; j < CPW; ++j) {
+    const int blk = wave * CPW + j;
+    const bool isx = blk * 8 < BM;            // wave-uniform: a copy never straddles (BM % 8 == 0)
+    const int row = blk * 8 + (l >> 3) - (isx ? 0 : BM);
+    const int c = (l & 7) ^ swz(row);
+    const int feat = (row & ~31) + 8 * ((row & 15) >> 2) + 4 * ((row >> 4) & 1) + (row & 3);  // w_slot(feat) == row
+    off[j] = (uint32_t)((isx ? min(row, xmax) : min(feat, wmax)) * K + 8 * c) * 2u;
+    src[j] = isx ? X + m0 * K : W + (int64_t)n0 * K;
+  }
+  auto copy_chunk = [&](int q, int st) {
+    const int k0 = min(q, nk - 1) * BK;       // past the end: the last chunk again, into a stage nobody multiplies
+#pragma unroll
+    for (int j = 0; j < CPW; ++j)
+      dma16(off[j], src[j] + k0, lds0 + (uint32_t)(st * SBYTES + (wave * CPW + j) * 1024));
+  };
+
+  f4 acc[PN][2][TM];
+#pragma unroll
+  for (int p = 0; p < PN; ++p)
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+      for (int t = 0; t < TM; ++t) acc[p][tt][t] = zero4();
+
+  struct Frags {
+    h8 wa[PN][2], xb[TM];
+  };
+  const unsigned char* sx = stages + (wm * WM + r) * ROW;
+  const unsigned char* sw = stages + XBYTES + (wn * WN + r) * ROW;
+  const uint32_t lo0 = (uint32_t)((g ^ swz(r)) << 4), lo1 = lo0 ^ 64u;  // units g and 4 + g
+  auto read = [&](Frags& f, int st, uint32_t lo) {
+#pragma unroll
+    for (int p = 0; p < PN; ++p)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+        f.wa[p][tt] = *reinterpret_cast<const h8*>(sw + st * SBYTES + (32 * p + 16 * tt) * ROW + lo);
+#pragma unroll
+    for (int t = 0; t < TM; ++t) f.xb[t] = *reinterpret_cast<const h8*>(sx + st * SBYTES + 16 * t * ROW + lo);
+  };
+  auto mul = [&](const Frags& f) {
+#pragma unroll
+    for (int t = 0; t < TM; ++t)
+#pragma unroll
+      for (int p = 0; p < PN; ++p)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) acc[p][tt][t] = mfma32(f.wa[p][tt], f.xb[t], acc[p][tt][t]);
+  };
+
+#pragma unroll
+  for (int q = 0; q < NS; ++q) copy_chunk(q, q);
+  wait_copies<(NS - 1) * CPW>();
+  lds_barrier();
+  Frags f0, f1;
+  read(f0, 0, lo0);
+  int st = 0;
+  for (int q = 0; q < nk; ++q) {
+    read(f1, st, lo1);
+    __builtin_amdgcn_sched_barrier(0);
+    mul(f0);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_copies<(NS - 2) * CPW>();  // chunk q + 1 has landed (q + 2 .. q + NS - 1 may be in flight)
+    lds_barrier();
+    copy_chunk(q + NS, st);
+    st = st == NS - 1 ? 0 : st + 1;
+    read(f0, st, lo0);              // after the last chunk: a repeated one, read and never used
+    __builtin_amdgcn_sched_barrier(0);
+    mul(f1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  wait_copies<0>();  // no copy may land in LDS after the workgroup has left it
+
+  OT* Y = static_cast<OT*>(a.y);  // may alias a.residual (in-place residual add)
+#pragma unroll
+  for (int p = 0; p < PN; ++p) {
+    const int n = n0 + wn * WN + 32 * p + 8 * g;
+    if (n >= N) continue;
+    float bv[8];
+    load8_f16_to_f32(a.bias + n, bv);
+#pragma unroll
+    for (int t = 0; t < TM; ++t) {
+      const int64_t m = m0 + wm * WM + 16 * t + r;
+      if (m >= M) continue;
+      float v[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = acc[p][0][t][i] + bv[i];
+        v[4 + i] = acc[p][1][t][i] + bv[4 + i];
+      }
+      if constexpr (EPI == kEpiBiasGelu) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = gelu_erf(v[j]);
+      }
+      if constexpr (EPI == kEpiBias) q_scale8(a, n, v);
+      if constexpr (EPI == kEpiBiasResidual) {
+        float rv[8];
+        load8_f32(a.residual + m * N + n, rv);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] += rv[j];
+      }
+      store8(Y + m * N + n, v);
+    }
+  }
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int NS, int EPI, typename OT>
+static hipError_t launch_ring_tile(const LinearArgs& a, hipStream_t s) {
+  const int64_t grid = ((a.m + BM - 1) / BM) * ((a.n + BN - 1) / BN);
+  if (grid > 0x7fffffff) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((linear_ring_kernel<BM, BN, WAVES_M, WAVES_N, NS, EPI, OT>), dim3((unsigned)grid),
+                     dim3(64 * WAVES_M * WAVES_N), 0, s, a);
+  return hipGetLastError();
+}
+
+// Tiles of the ring kernel, and the model that picks one: a CU works through
+// ceil(tiles / 256) tiles of (K / 64) * step + end each, after a fixed start (launch, first
+// copies, last stores).  step / end / start in units of 10 ns, fitted to sweeps on MI355X
+// over 22 shapes from 3 x 2048 x 1536 to 32768 x 2048 x 512 (the tile it picks was within
+// 15 % of the fastest on each): a 128 x 128 tile alone takes 0.5 us per 64 k values, a
+// 32 x 32 one 0.1 us, and the ends cost 0.7-1.7 us of stores and epilogue per tile.
+struct RingTile {
+  int bm, bn, step, end, start;
+};
+constexpr RingTile kRingTiles[] = {
+    {128, 128, 50, 170, 550}, {128, 64, 27, 130, 400}, {64, 64, 15, 100, 330}, {32, 64, 10, 75, 270}, {32, 32, 10, 70, 250},
+};
+
+static int ring_tile(int64_t m, int n, int k) {
+  int best = 0;
+  int64_t best_cost = INT64_MAX;
+  for (int i = 0; i < (int)(sizeof(kRingTiles) / sizeof(kRingTiles[0])); ++i) {
+    const RingTile& t = kRingTiles[i];
+    const int64_t tiles = ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+    const int64_t cost = t.start + ((tiles + 255) / 256) * ((int64_t)(k / 64) * t.step + t.end);
+    if (cost < best_cost) best_cost = cost, best = i;
+  }
+  return best;
+}
+
+// Whether a call of the built-in choice `variant` runs the ring kernel instead: FP16 X with
+// K % 64 == 0, where the choice is one of linear_kernel's tiles (1-4), or variant 8 with
+// K >= 2048.  There the 256 x 256 ring tile's 64-wide chunks win what its missing overlap of
+// tile ends loses: 32768 x 512 x 2048 with residual 81.5 vs 84 us, 8192^3 932 vs 1206 us; at
+// K = 1024 variant 8 is ahead, 310 vs 321 us for 32768 x 4096 with GELU.
+constexpr int kRing256MinK = 2048;
+static bool ring_applies(int variant, int k) {
+  return k % 64 == 0 && k <= (1 << 20) && (variant <= 4 || (variant == 8 && k >= kRing256MinK));
+}
+
+template <int EPI, typename OT>
+static hipError_t launch_ring(int variant, const LinearArgs& a, hipStream_t s) {
+  if (variant == 8) return launch_ring_tile<256, 256, 2, 4, 2, EPI, OT>(a, s);
+  switch (ring_tile(a.m, a.n, a.k)) {
+    case 0: return launch_ring_tile<128, 128, 2, 2, 2, EPI, OT>(a, s);
+    case 1: return launch_ring_tile<128, 64, 2, 2, 3, EPI, OT>(a, s);
+    case 2: return launch_ring_tile<64, 64, 2, 2, 5, EPI, OT>(a, s);
+    case 3: return launch_ring_tile<32, 64, 2, 2, 6, EPI, OT>(a, s);
+    default: return launch_ring_tile<32, 32, 2, 1, 10, EPI, OT>(a, s);
+  }
+}
+
 // ---- X-stationary projection (FP16 X, K = 128 or 256, N % 64 == 0) ----
 // For projections with a short K (the d_model-256 QKV projection: 262,144 x 768 x 256),
 // each wave keeps its 32 tokens' whole X rows as MFMA fragments in registers (K = 256:
@@ -1294,6 +1512,12 @@ static hipError_t launch_linear(const LinearArgs& a, hipStream_t s) {
 //      N % 64 == 0, bias / GELU epilogues; other inputs run 8)
 template <typename XT, int EPI, typename OT>
 static hipError_t linear_variant(int variant, const LinearArgs& a, hipStream_t s) {
+  if (variant == 0) {  // the built-in choice
+    variant = mpk_linear_auto_variant(a.m, a.n, a.k);
+    if constexpr (std::is_same<XT, _Float16>::value) {
+      if (ring_applies(variant, a.k)) return launch_ring<EPI, OT>(variant, a, s);
+    }
+  }
   switch (variant) {
     case 1: return launch_linear<128, 128, 64, 2, XT, EPI, OT>(a, s);
     case 2: return launch_linear<128, 64, 64, 4, XT, EPI, OT>(a, s);
@@ -1369,7 +1593,6 @@ extern "C" int mpk_linear(const void* x, int x_dtype, const void* w, const void*
   if (n % 8 != 0 || k % 8 != 0) return MPK_EUNSUPPORTED;
   if (!aligned16(x) || !aligned16(w) || !aligned16(b) || !aligned16(y)) return MPK_EALIGN;
   if (m == 0) return MPK_OK;
-  if (variant == 0) variant = mpk_linear_auto_variant(m, n, k);
   LinearArgs a{};
   a.x = x; a.w = static_cast<const _Float16*>(w); a.bias = static_cast<const _Float16*>(b); a.y = y;
   a.m = m; a.n = n; a.k = k;
@@ -1398,7 +1621,6 @@ extern "C" int mpk_linear_qscaled(const void* x, int x_dtype, const void* w, con
   if (n % 8 != 0 || k % 8 != 0 || q_cols % 8 != 0) return MPK_EUNSUPPORTED;
   if (!aligned16(x) || !aligned16(w) || !aligned16(b) || !aligned16(y)) return MPK_EALIGN;
   if (m == 0) return MPK_OK;
-  if (variant == 0) variant = mpk_linear_auto_variant(m, n, k);
   LinearArgs a{};
   a.x = x; a.w = static_cast<const _Float16*>(w); a.bias = static_cast<const _Float16*>(b); a.y = y;
   a.m = m; a.n = n; a.k = k;
@@ -1452,7 +1674,6 @@ extern "C" int mpk_linear_residual(const void* x, int x_dtype, const void* w, co
   if (n % 8 != 0 || k % 8 != 0) return MPK_EUNSUPPORTED;
   if (!aligned16(x) || !aligned16(w) || !aligned16(b) || !aligned16(residual) || !aligned16(y)) return MPK_EALIGN;
   if (m == 0) return MPK_OK;
-  if (variant == 0) variant = mpk_linear_auto_variant(m, n, k);
   LinearArgs a{};
   a.x = x; a.w = static_cast<const _Float16*>(w); a.bias = static_cast<const _Float16*>(b); a.y = y;
   a.residual = residual; a.m = m; a.n = n; a.k = k;
