@@ -528,6 +528,52 @@ def test_fp16_causal_attention_32x32(hip_device, b, h, s, hd, variant):
     _close(out, _ref_attention(q, k, v, scale, True), 3e-3, 3e-3, "fp16 causal attention (32x32)")
 
 
+@pytest.mark.parametrize(
+    "b,h,s,hd,io",
+    [(24, 8, 257, 128, torch.float16), (6, 16, 581, 128, torch.float16), (16, 8, 400, 128, torch.float32),
+     (32, 8, 256, 256, torch.float16), (13, 8, 640, 256, torch.float16)],
+)
+@pytest.mark.parametrize("causal", [True, False])
+def test_attention_32x32_wide_heads(hip_device, b, h, s, hd, io, causal):
+    """Head dims 128 / 256 on the 32x32 kernel (swizzled K / V tiles), as variant 0 picks it from
+    256 keys and 49,152 / 65,536 queries: ragged lengths, negative scale, key mask."""
+    from tiktoktechjam2026_amd.custom_kernel.hip_attention import attention
+
+    print(f"\n[attention 32x32 wide] b={b} h={h} s={s} hd={hd} {io} causal={causal}", flush=True)
+    _, q, k, v = _packed_qkv(b, s, h, hd, 79, hip_device, io)
+    rows = [0, b - 1]
+    for scale in (hd ** -0.5, -(hd ** -0.5)):
+        out = attention(q, k, v, scale, causal=causal)
+        _close(out[rows], _ref_attention(q[rows], k[rows], v[rows], scale, causal), 3e-3, 3e-3, "wide heads")
+    mask = torch.rand(b, s, generator=torch.Generator().manual_seed(5)) > 0.3
+    mask[0] = torch.arange(s) < s // 2
+    mask[:, 0] = True
+    out = attention(q, k, v, scale, causal=causal, key_valid=mask.to(hip_device))
+    _close(out[rows], _ref_attention(q[rows], k[rows], v[rows], scale, causal, mask[rows]), 3e-3, 3e-3, "masked")
+
+
+@pytest.mark.parametrize("hd,variant", [(8, 1), (16, 2), (16, 5), (32, 1), (32, 6), (32, 7), (64, 6), (64, 8), (128, 1), (256, 1)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_attention_key_mask_ranges(hip_device, hd, variant, causal):
+    """Key masks by where their valid keys lie: padded tails ending inside a tile, on its edge and one
+    key past it, a masked head, holes, a single valid key, none.  Rows that see no valid key give zeros."""
+    from tiktoktechjam2026_amd.custom_kernel.hip_attention import attention
+
+    s = 331
+    pos = torch.arange(s)
+    masks = [pos < n for n in (s, 1, 63, 64, 65, 128, 129, 192, 300)]
+    masks += [pos >= 70, pos >= 64, (pos % 3 != 0), (pos < 64) | (pos > 200), pos == 150, pos < 0]
+    mask = torch.stack(masks)
+    b = len(masks)
+    _, q, k, v = _packed_qkv(b, s, 2, hd, 83, hip_device, torch.float16)
+    out = attention(q, k, v, hd ** -0.5, causal=causal, key_valid=mask.to(hip_device), variant=variant).cpu()
+    visible = mask[:, None, :] & (torch.ones(s, s, dtype=torch.bool).tril() if causal else torch.ones(s, s, dtype=torch.bool))
+    seen = visible.any(-1)
+    ref = _ref_attention(q, k, v, hd ** -0.5, causal, mask)
+    _close(out[seen], ref[seen], 3e-3, 3e-3, "key mask")
+    assert torch.equal(out[~seen], torch.zeros_like(out[~seen]))
+
+
 @pytest.mark.parametrize("variant", [6, 7, 8])
 def test_attention_32x32_noncausal_fp32io_keymask_negative_scale(hip_device, variant):
     from tiktoktechjam2026_amd.custom_kernel.hip_attention import attention

@@ -94,6 +94,32 @@ __device__ float wg_absmax(const float* base, int64_t row_stride, int rows, int 
   return r;
 }
 
+// Valid-key range of a mask row, for keys [0, kv_end): first_bad = the first key that may not be
+// attended (kv_end or more if there is none), last_ok = one past the last key that may.  Keys
+// below first_bad need no mask and keys from last_ok on contribute nothing, so for a
+// right-padded sequence only the tile that holds its end pays for the mask and the padded
+// tiles are not read at all.  The waves test 64 keys per ballot; every thread must call it
+// (range: two ints of LDS).
+template <int NW>
+__device__ void mask_range(const uint8_t* valid, int kv_end, int* range, int& first_bad, int& last_ok) {
+  const int l = threadIdx.x & 63;
+  if (threadIdx.x == 0) range[0] = kv_end, range[1] = 0;
+  __syncthreads();
+  int fb = kv_end, lk = 0;
+  for (int k0 = 64 * wave_id(); k0 < kv_end; k0 += 64 * NW) {
+    const uint64_t ok = __builtin_amdgcn_ballot_w64(k0 + l < kv_end && valid[min(k0 + l, kv_end - 1)] != 0);
+    if (~ok) fb = min(fb, k0 + (int)__builtin_ctzll(~ok));
+    if (ok) lk = k0 + 64 - (int)__builtin_clzll(ok);
+  }
+  if (l == 0) {
+    atomicMin(&range[0], fb);
+    atomicMax(&range[1], lk);
+  }
+  __syncthreads();
+  first_bad = __builtin_amdgcn_readfirstlane(range[0]);
+  last_ok = __builtin_amdgcn_readfirstlane(range[1]);
+}
+
 struct AttnArgs {
   const void* q;
   const void* k;
@@ -169,7 +195,14 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(AttnArgs a) {
   const int qw0 = q0 + wave * 16 * QT;       // first query of this wave
   const int qw_last = qw0 + 16 * QT - 1;     // last query of this wave
 
-  const int kv_end = a.causal ? min(q0 + QB, S) : S;  // keys [0, kv_end) can matter
+  int kv_end = a.causal ? min(q0 + QB, S) : S;  // keys [0, kv_end) can matter
+  int first_bad = S;                            // keys [0, first_bad) need no mask
+  if constexpr (KEYMASK) {
+    __shared__ int range[2];
+    int last_ok;
+    mask_range<NW>(kv_valid, kv_end, range, first_bad, last_ok);
+    kv_end = max(1, min(kv_end, last_ok));
+  }
   const int ntiles = (kv_end + KTILE - 1) / KTILE;
 
   // FP32 inputs: power-of-two exponents for K and V over the keys this workgroup reads
@@ -366,18 +399,18 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(AttnArgs a) {
 
   // ---- one key tile: S^T, online softmax, O^T += V^T P^T ----
   // FIRST: the tile may hold a row's first visible key, so rows can still be
-  // "fresh" (their scores were computed without the -mrow offset).  Without a
-  // key mask every row sees key 0, so only tile 0 needs that handling and the
-  // steady-state tiles skip it.
+  // "fresh" (their scores were computed without the -mrow offset).  Where key 0
+  // is valid every row sees it, so only tile 0 needs that handling and the
+  // tiles after it skip it; with a key mask, all tiles do if tile 0 holds a masked key.
   auto process = [&](const int kb, const _Float16* ksb, const _Float16* vtb, const float* kbb, auto first_tag) {
-    constexpr bool MAYBE_FRESH = decltype(first_tag)::value || KEYMASK;
+    constexpr bool MAYBE_FRESH = decltype(first_tag)::value;
     if (a.causal && kb > qw_last) return;  // whole tile is in this wave's future
     // Key pairs [0, npv) hold keys visible to some query of this wave; in a
     // causal tile on the diagonal only the last of them straddles it (queries of
     // a wave are 16-aligned, pairs 32-aligned) and the pairs after it are skipped.
     const int npv = a.causal ? min(NP, (qw_last - kb) / 32 + 1) : NP;
     const bool need_causal = a.causal && kb + 32 * npv - 1 > qw0;  // last visible pair straddles the diagonal
-    const bool need_bias = KEYMASK || kb + KTILE > S;               // padded keys or keys past the end
+    const bool need_bias = kb + KTILE > first_bad;                  // masked keys or keys past the end
 
     // S^T = K (Q*c)^T - m for the visible key pairs x 16*QT queries
     f4 sc[NP][2][QT];  // [key pair][tile in pair][q tile]
@@ -554,8 +587,8 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(AttnArgs a) {
     const int cur = tile & 1;
     const bool more = tile + 1 < ntiles;
     if (more) fetch((tile + 1) * KTILE);
-    if (tile == 0)
-      process(0, ks_lds[cur], vt_lds[cur], kbias[cur], std::true_type{});
+    if (tile == 0 || (KEYMASK && first_bad < KTILE))
+      process(tile * KTILE, ks_lds[cur], vt_lds[cur], kbias[cur], std::true_type{});
     else
       process(tile * KTILE, ks_lds[cur], vt_lds[cur], kbias[cur], std::false_type{});
     if (more) stash(cur ^ 1);
@@ -598,7 +631,7 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// 32x32 variant for head_dim 32 / 64: S^T = K Q^T and O^T = V^T P^T on
+// 32x32 kernel for head dims 32 to 256: S^T = K Q^T and O^T = V^T P^T on
 // v_mfma_f32_32x32x16_f16, whose long issue-to-result time lets the softmax
 // VALU work of the same wave run beside it (the 16x16x32 form leaves little
 // room for that, and at these head dims the softmax is the larger cost).
@@ -629,7 +662,7 @@ template <int HD, int NW, int KTILE, typename IT, typename OT, bool KEYMASK, boo
 // (four waves per SIMD, i.e. at most 128 VGPRs, for FP16 input at head dim 32 with 64-key
 // tiles; FP32 input carries a per-row score factor, one register more, and runs at three)
 __global__ __launch_bounds__(64 * NW) __attribute__((
-    amdgpu_waves_per_eu(HD == 32 && KTILE == 64 && std::is_same<IT, _Float16>::value ? 4 : 1)))
+    amdgpu_waves_per_eu(HD == 32 && KTILE == 64 && std::is_same<IT, _Float16>::value ? 4 : HD >= 128 ? 2 : 1)))
 void attention32_kernel(AttnArgs a) {
   static_assert(!PS || std::is_same<IT, _Float16>::value, "pre-scaled q is FP16");
   constexpr int NT = 64 * NW;
@@ -638,10 +671,17 @@ void attention32_kernel(AttnArgs a) {
   constexpr int NB = KTILE / 32;  // 32-key blocks per tile
   constexpr int QS = HD / 16;     // 16-wide head-dim steps of S^T
   constexpr int DT = HD / 32;     // 32-row head-dim tiles of O^T
-  static_assert(HD == 32 || HD == 64, "head dim");
+  static_assert(HD == 32 || HD == 64 || HD == 128 || HD == 256, "head dim");
   static_assert(KTILE % 32 == 0 && KTILE <= NT, "key tile");
 
-  __shared__ __align__(16) _Float16 ks_lds[2][SH::KBUF];
+  // Head dims 128 and 256: unpadded rows with their 16-byte units permuted instead, which
+  // keeps the tiles at 16 KB each (two workgroups per CU): K's unit u of key row R sits in
+  // slot u ^ (R % 16), so the 16-lane phases of a fragment read (whose rows are distinct
+  // mod 16 after kappa32) cover all banks; V's in slot u ^ 4 (R % 4), so the four key rows
+  // of a transpose read fall into different 64-byte bank groups.
+  constexpr bool SWZ = HD >= 128;
+  constexpr int LDK = SWZ ? HD : SH::LDK;
+  __shared__ __align__(16) _Float16 ks_lds[2][KTILE * LDK];
   // V is staged row-major like K (one 16-byte store per chunk); the P V product
   // reads its V^T fragments with LDS transpose loads (ds_read_b64_tr_b16).  Each
   // 32-lane half of such a read covers 4 consecutive keys x 64 bytes of head dims,
@@ -650,7 +690,7 @@ void attention32_kernel(AttnArgs a) {
   // 16-byte-padded stride, right for the K fragment reads, conflicts two ways here):
   // unpadded rows at hd 32.  (At hd 64 that takes 192-byte rows, which measured no
   // faster than the K stride; hd 64 keeps it.)
-  constexpr int LDVR = HD == 32 ? HD : SH::LDK;
+  constexpr int LDVR = HD == 32 || SWZ ? HD : SH::LDK;
   __shared__ __align__(16) _Float16 vr_lds[2][KTILE * LDVR];
   __shared__ float kbias[2][KTILE];
 
@@ -701,7 +741,14 @@ void attention32_kernel(AttnArgs a) {
   const int q = qw0 + qi;
   const int trow = kappa32(qi);    // tile row this lane feeds as an A-operand row
 
-  const int kv_end = a.causal ? min(q0 + QB, S) : S;
+  int kv_end = a.causal ? min(q0 + QB, S) : S;
+  int first_bad = S;  // keys [0, first_bad) need no mask
+  if constexpr (KEYMASK) {
+    __shared__ int range[2];
+    int last_ok;
+    mask_range<NW>(kv_valid, kv_end, range, first_bad, last_ok);
+    kv_end = max(1, min(kv_end, last_ok));
+  }
   const int ntiles = (kv_end + KTILE - 1) / KTILE;
 
   // FP32 inputs: power-of-two exponents for K and V over the keys this workgroup reads,
@@ -812,8 +859,8 @@ void attention32_kernel(AttnArgs a) {
   h8 kreg[SH::PER_THREAD], vreg[SH::PER_THREAD];
   float breg = 0.f;
   // Key bias (-inf for masked keys and keys past the sequence end): staged only for
-  // tiles that read it, which is every tile with a key mask and otherwise only a tile
-  // that runs past the sequence end (wave-uniform).
+  // tiles that read it, those that reach the first masked key or run past the sequence
+  // end (wave-uniform).
   bool bias_staged = false;
   const uint32_t krow_bytes = (uint32_t)(a.ks[2] * (int64_t)sizeof(IT));
   const uint32_t vrow_bytes = (uint32_t)(a.vs[2] * (int64_t)sizeof(IT));
@@ -824,8 +871,11 @@ void attention32_kernel(AttnArgs a) {
   // other vector-memory operation) before its barrier.  Measured on MI355X in one process,
   // outputs bit-identical: cfg5 forward 48.61-48.63 vs 49.03-49.06 ms, cfg2 level; at head
   // dim 64 (cfg4) the register staging below stays, 2.594 vs 2.603 ms.
-  constexpr bool DMA_KV = !F32IN && HD == 32;
-  constexpr int KUP = SH::LDK / 8, VUP = LDVR / 8, KU = HD / 8;
+  constexpr bool DMA_KV = !F32IN && HD != 64;
+  constexpr int KUP = LDK / 8, VUP = LDVR / 8, KU = HD / 8;
+  // slot of 16-byte unit u of key row `key` (its own inverse), see SWZ
+  auto kslot = [](int key, int u) { return SWZ ? u ^ (key & 15) : u; };
+  auto vslot = [](int key, int u) { return SWZ ? u ^ ((key & 3) << 2) : u; };
   constexpr int KCOPIES = KTILE * KUP / 64, VCOPIES = KTILE * VUP / 64;
   static_assert(!DMA_KV || (KTILE * KUP % 64 == 0 && KTILE * VUP % 64 == 0), "whole copies");
   auto fetch_dma = [&](int kb, int buf) {
@@ -836,14 +886,14 @@ void attention32_kernel(AttnArgs a) {
     const _Float16* vbase = reinterpret_cast<const _Float16*>(Vp) + (int64_t)kb * a.vs[2];
     for (int j = wave; j < KCOPIES + VCOPIES; j += NW) {
       if (j < KCOPIES) {
-        const int u = 64 * j + l, key = min(u / KUP, last), pos = u % KUP;
+        const int u = 64 * j + l, key = min(u / KUP, last), pos = kslot(u / KUP, u % KUP);
         dma16((uint32_t)key * krow_bytes + (pos < KU ? 16u * pos : 0u), kbase, (uint32_t)__builtin_amdgcn_readfirstlane((int)(kl + 1024u * j)));
       } else {
-        const int u = 64 * (j - KCOPIES) + l, key = min(u / VUP, last), pos = u % VUP;
+        const int u = 64 * (j - KCOPIES) + l, key = min(u / VUP, last), pos = vslot(u / VUP, u % VUP);
         dma16((uint32_t)key * vrow_bytes + (pos < KU ? 16u * pos : 0u), vbase, (uint32_t)__builtin_amdgcn_readfirstlane((int)(vl + 1024u * (j - KCOPIES))));
       }
     }
-    bias_staged = KEYMASK || kb + KTILE > S;
+    bias_staged = kb + KTILE > first_bad;
     if (bias_staged && threadIdx.x < KTILE) {
       const int gk = kb + threadIdx.x;
       bool valid = gk < S;
@@ -875,7 +925,7 @@ void attention32_kernel(AttnArgs a) {
         else vreg[i] = buffer_load8_as_half(vr, off, Vp);
       }
     }
-    bias_staged = KEYMASK || kb + KTILE > S;
+    bias_staged = kb + KTILE > first_bad;
     if (bias_staged && threadIdx.x < KTILE) {
       const int gk = kb + threadIdx.x;
       bool valid = gk < S;
@@ -889,8 +939,8 @@ void attention32_kernel(AttnArgs a) {
       const int cc = threadIdx.x + i * NT;
       if (cc < SH::CHUNKS) {
         const int key = cc / SH::CPK, col = (cc % SH::CPK) * 8;
-        *reinterpret_cast<h8*>(&ks_lds[buf][key * SH::LDK + col]) = kreg[i];
-        *reinterpret_cast<h8*>(&vr_lds[buf][key * LDVR + col]) = vreg[i];
+        *reinterpret_cast<h8*>(&ks_lds[buf][key * LDK + 8 * kslot(key, col / 8)]) = kreg[i];
+        *reinterpret_cast<h8*>(&vr_lds[buf][key * LDVR + 8 * vslot(key, col / 8)]) = vreg[i];
       }
     }
     if (bias_staged && threadIdx.x < KTILE) kbias[buf][threadIdx.x] = breg;
@@ -905,7 +955,8 @@ void attention32_kernel(AttnArgs a) {
   const int vtr_r = l & 15, vtr_g = l >> 4, vtr_q = vtr_r & 3;
   const int vtr_dim = 16 * (vtr_g & 1) + 8 * (vtr_q & 1) + 4 * (vtr_q >> 1);
   auto vt_frag = [&](const _Float16* vrb, int dt, int k0) {
-    const _Float16* p0 = vrb + (k0 + (vtr_r >> 2)) * LDVR + 32 * dt + vtr_dim;
+    const _Float16* p0 = vrb + (k0 + (vtr_r >> 2)) * LDVR +
+                         (SWZ ? (32 * dt) ^ ((vtr_r >> 2) << 5) : 32 * dt) + vtr_dim;
     const s4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)(p0));
     const s4v hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s4v*)(p0 + 4 * LDVR));
     typedef _Float16 h4v __attribute__((ext_vector_type(4)));
@@ -919,6 +970,11 @@ void attention32_kernel(AttnArgs a) {
     return v;
   };
 
+  // K fragment (A operand of S^T): tile row 32 nb + trow, head dims 16 st + 8 hf .. +7
+  auto k_frag = [&](const _Float16* ksb, int nb, int st) {
+    return *reinterpret_cast<const h8*>(&ksb[(32 * nb + trow) * LDK + 8 * kslot(trow, 2 * st + hf)]);
+  };
+
   // ---- one key tile ----
   // The S^T products of all of the tile's 32-key blocks are issued first; the
   // softmax and P V of block nb then run on the VALU while the MFMAs of the
@@ -928,12 +984,12 @@ void attention32_kernel(AttnArgs a) {
   // past the sequence end or masked keys; steady-state tiles skip those checks.
   auto process = [&](const int kb, const _Float16* ksb, const _Float16* vtb, const float* kbb, auto first_tag,
                      auto edge_tag) {
-    constexpr bool MAYBE_FRESH = decltype(first_tag)::value || KEYMASK;
     constexpr bool EDGE = decltype(edge_tag)::value;
+    constexpr bool MAYBE_FRESH = decltype(first_tag)::value || (KEYMASK && EDGE);
     // blocks [0, nbv) hold keys visible to some query of the wave (wave-uniform)
     const int nbv = (EDGE && a.causal) ? min(NB, (qw0 - kb) / 32 + 1) : NB;
     if (EDGE && nbv <= 0) return;
-    const bool need_bias = KEYMASK || kb + KTILE > S;
+    const bool need_bias = kb + KTILE > first_bad;
 
     // S^T (32 keys x 32 queries) per block, raw scores (pre-scaled steady tiles: minus m)
     constexpr bool STEADY = !EDGE && !MAYBE_FRESH && HD == 32 && KTILE == 64;
@@ -975,8 +1031,7 @@ void attention32_kernel(AttnArgs a) {
       }
 #pragma unroll
       for (int st = 0; st < QS; ++st) {
-        const h8 ka = *reinterpret_cast<const h8*>(&ksb[(32 * nb + trow) * SH::LDK + 16 * st + 8 * hf]);
-        sc[nb] = mfma32x32(ka, qf[st], sc[nb]);
+        sc[nb] = mfma32x32(k_frag(ksb, nb, st), qf[st], sc[nb]);
       }
     }
     if constexpr (EDGE) {
@@ -1104,8 +1159,7 @@ void attention32_kernel(AttnArgs a) {
           sc[nb] = f16v{};
 #pragma unroll
           for (int st = 0; st < QS; ++st) {
-            const h8 ka = *reinterpret_cast<const h8*>(&ksb[(32 * nb + trow) * SH::LDK + 16 * st + 8 * hf]);
-            sc[nb] = mfma32x32(ka, qf[st], sc[nb]);
+            sc[nb] = mfma32x32(k_frag(ksb, nb, st), qf[st], sc[nb]);
           }
         }
         raise_max();
@@ -1195,7 +1249,8 @@ void attention32_kernel(AttnArgs a) {
     __syncthreads();
   };
   auto step = [&](int tile, auto first_tag, auto edge_tag) { step_in(tile, tile & 1, first_tag, edge_tag); };
-  const int steady_end = KEYMASK ? 1 : max(1, min(ntiles, (a.causal ? min(q0, S) : S) / KTILE));
+  // (with a key mask: and below the first masked key; if tile 0 holds one, none)
+  const int steady_end = max(1, min(ntiles, min(a.causal ? q0 : S, first_bad) / KTILE));
 
   if constexpr (DMA_KV) {
     fetch_dma(0, 0);
@@ -1312,8 +1367,40 @@ static hipError_t attn32_variant(int variant, const AttnArgs& a, hipStream_t s) 
   }
 }
 
+// The built-in choice (variant 0).  mpk_attention_auto_variant answers by sequence length and
+// head dim; here batch, direction and mask refine it.  n8: 256-query workgroups of the launch.
+// Measured on MI355X (B x H x S, us, FP16 I/O; c: causal, f: full, p: full with a key mask of
+// right-padded rows, half of them padding at most):
+//   head dim 128 / 256, the 16x16 kernel -> 32x32 with 8 waves (one LDS fragment serves 32
+//   queries instead of 16, and no hi + lo split of q doubles the S^T products):
+//     256 x 1024, hd 128: c 167 -> 115, f 309 -> 174    256 x 512, hd 128: c 55 -> 44, f 86 -> 54
+//     256 x 512, hd 256: c 102 -> 94, f 163 -> 101      64 x 1024, hd 256: c 75 -> 78, f 123 -> 81
+//   but 16 x 2048 hd 128: c 56 -> 64, f 69 -> 65 and 16 x 1024: c 26 -> 35 (too few 256-query
+//   workgroups), and 256 x 128: 9.1 -> 9.9; so from 256 keys and 49,152 queries (hd 256: 65,536).
+//   FP32 I/O at head dim 256 spills there and stays on the 16x16 kernel.
+//   head dims 32 / 64, 4 -> 8 waves: hd 32 256 x 2000 c 121 -> 119, f 229 -> 200, p 185 -> 172;
+//     hd 64 256 x 1500 c 114 -> 108, f 202 -> 186, p 169 -> 197; 8 x 900 f 16.6 -> 22.7,
+//     64 x 512 c 13.5 -> 15.9: 8 waves where at least 512 workgroups remain.
+static int attn_builtin(const AttnArgs& a, int hd, bool f32_in) {
+  const int v = mpk_attention_auto_variant(a.batch, a.heads, a.seq, hd);
+  const int64_t rows = (int64_t)a.batch * a.heads, n8 = rows * ((a.seq + 255) / 256);
+  if (hd >= 128) return a.seq >= 256 && rows * a.seq >= (hd == 128 ? 49152 : 65536) && !(f32_in && hd == 256) ? 7 : v;
+  if (f32_in || a.seq < 256 || hd < 32) return v;
+  if (hd == 32) return v == 7 || (!a.causal && n8 >= 512) ? 7 : 6;
+  return !a.key_valid && n8 >= 512 && (v == 7 || !a.causal) ? 7 : 6;
+}
+
 template <typename IT, typename OT>
 static hipError_t attn_dispatch(int variant, const AttnArgs& a, int hd, hipStream_t s) {
+  constexpr bool F32IN = std::is_same<IT, float>::value;
+  if (variant == 0) {
+    variant = attn_builtin(a, hd, F32IN);
+    // (not among the variants that can be pinned at these head dims)
+    if (variant == 7 && hd == 128) return launch_attn32<128, 8, 64, IT, OT>(a, s);
+    if constexpr (!F32IN) {
+      if (variant == 7 && hd == 256) return launch_attn32<256, 8, 32, IT, OT>(a, s);
+    }
+  }
   if (variant >= 6) {
     if (hd == 32) return attn32_variant<32, IT, OT>(variant, a, s);
     if (hd == 64) return attn32_variant<64, IT, OT>(variant, a, s);
@@ -1369,8 +1456,7 @@ extern "C" int mpk_causal_attention(const void* q, const void* k, const void* v,
       if ((st[i][j] * esz) % 16 != 0) return MPK_EALIGN;
   }
   if (batch == 0 || seq_len == 0) return MPK_OK;
-  if (variant == 0) variant = mpk_attention_auto_variant(batch, heads, seq_len, head_dim);
-  if (variant < 1 || variant > 8) return MPK_EUNSUPPORTED;
+  if (variant < 0 || variant > 8) return MPK_EUNSUPPORTED;
   AttnArgs a{};
   a.q = q; a.k = k; a.v = v; a.o = o;
   for (int j = 0; j < 4; ++j) {
@@ -1411,7 +1497,8 @@ extern "C" int mpk_causal_attention_prescaled(const void* q, const void* k, cons
   if (variant == 0) {
     const int64_t rows = (int64_t)batch * heads, nqb8 = ((int64_t)seq_len + 255) / 256;
     const bool grouped8 = rows % 64 == 0 && (rows / 8) * nqb8 >= 1024;
-    variant = head_dim == 32 ? (grouped8 ? 7 : 6) : (seq_len < 1024 ? 7 : 6);
+    // (full attention from 512 workgroups: as attn_builtin)
+    variant = head_dim == 32 ? (grouped8 || (!causal && rows * nqb8 >= 512) ? 7 : 6) : (seq_len < 1024 ? 7 : 6);
   }
   if (variant < 6 || variant > 8) return MPK_EUNSUPPORTED;
   const int64_t* st[4] = {q_strides, k_strides, v_strides, o_strides};
