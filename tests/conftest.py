@@ -23,7 +23,7 @@ def pytest_configure(config):
 def _ensure_library_built() -> None:
     from tiktoktechjam2026_amd import build
 
-    if not os.path.exists(build.LIB_PATH):
+    if not (os.path.exists(build.LIB_PATH) and os.path.exists(build.OPS_PATH)):
         build.build(verbose=True)
 
 

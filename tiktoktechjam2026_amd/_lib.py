@@ -14,7 +14,7 @@ from typing import Optional
 
 import torch
 
-from .build import LIB_PATH
+from .build import LIB_PATH, OPS_PATH
 
 F32 = 0
 F16 = 1
@@ -160,6 +160,23 @@ def load() -> ctypes.CDLL:
                 fn.argtypes = argtypes
             _lib = lib
     return _lib
+
+
+_ops_loaded = False
+
+
+def load_ops() -> None:
+    """Load ``libmpk_ops.so`` once: the GPU kernels of the ``mpk::`` torch operators."""
+    global _ops_loaded
+    load()
+    with _lock:
+        if not _ops_loaded:
+            if not os.path.exists(OPS_PATH):
+                raise RuntimeError(
+                    f"{OPS_PATH} is missing: build it first (python -m tiktoktechjam2026_amd.build)"
+                )
+            torch.ops.load_library(OPS_PATH)
+            _ops_loaded = True
 
 
 def check(status: int, what: str) -> None:

@@ -1,4 +1,5 @@
-"""Compile the gfx950 HIP sources into the in-tree C-ABI library ``libmpk.so``.
+"""Compile the gfx950 HIP sources into the in-tree C-ABI library ``libmpk.so``, and the torch
+operators' host code (``csrc/torch_ops.cpp``) into ``libmpk_ops.so`` beside it.
 
     python -m tiktoktechjam2026_amd.build          # build (always recompiles)
 
@@ -24,6 +25,8 @@ CSRC_DIR = os.path.join(PKG_DIR, "csrc")
 INCLUDE_DIR = os.path.join(REPO_DIR, "include")
 BUILD_DIR = os.path.join(PKG_DIR, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libmpk.so")
+OPS_SOURCE = os.path.join(CSRC_DIR, "torch_ops.cpp")
+OPS_PATH = os.path.join(PKG_DIR, "libmpk_ops.so")
 
 ARCH = "gfx950"
 COMMON_FLAGS = [
@@ -77,19 +80,56 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_ops() -> str:
+    """Host-only C++ against torch's headers."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    obj = os.path.join(BUILD_DIR, "torch_ops.o")
+    cmd = [
+        _hipcc(), "-x", "c++", "-std=c++17", "-O2", "-fPIC", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+        f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE_DIR}",
+        f"-I{os.path.join(root, 'include')}", f"-I{os.path.join(root, 'include', 'torch', 'csrc', 'api', 'include')}",
+        "-I" + os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"), "-c", OPS_SOURCE, "-o", obj,
+    ]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"hipcc failed for torch_ops.cpp:\n{proc.stdout}")
+    return obj
+
+
+def _link_ops(obj: str) -> None:
+    """``libmpk_ops.so`` finds ``libmpk.so`` beside itself."""
+    import torch
+
+    tmp = OPS_PATH + ".tmp"
+    cmd = [
+        _hipcc(), "-shared", "-fPIC", obj, "-o", tmp, f"-L{PKG_DIR}", "-l:" + os.path.basename(LIB_PATH),
+        f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip",
+        "-Wl,-rpath,$ORIGIN",
+    ]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link of libmpk_ops.so failed:\n{proc.stdout}")
+    os.replace(tmp, OPS_PATH)
+
+
 def build(verbose: bool = True) -> str:
-    """Compile every HIP source and link ``libmpk.so``; returns the library path."""
+    """Compile every source and link ``libmpk.so`` and ``libmpk_ops.so``; returns the former's path."""
     os.makedirs(BUILD_DIR, exist_ok=True)
     srcs = sources()
     jobs = max(1, min(len(srcs), int(os.environ.get("MAX_JOBS", os.cpu_count() or 4)), 16))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        ops_obj = pool.submit(_compile_ops)
         objs = list(pool.map(_compile, srcs))
+        ops_obj = ops_obj.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp]
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link of libmpk.so failed:\n{proc.stdout}")
     os.replace(tmp, LIB_PATH)
+    _link_ops(ops_obj)
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} HIP sources for {ARCH}")
     return LIB_PATH

@@ -48,11 +48,10 @@ def _layout_ok(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, dtype: torch.d
         return False
     if q.shape[-1] not in HEAD_DIMS:
         return False
-    if not (q.stride(-1) == k.stride(-1) == v.stride(-1) == 1):
-        return False
-    esz = q.element_size()
+    unit = 16 // q.element_size()  # rows start on 16-byte boundaries
     for t in (q, k, v):
-        if any((s * esz) % 16 != 0 for s in t.stride()[:3]):
+        s0, s1, s2, s3 = t.stride()
+        if s3 != 1 or s0 % unit or s1 % unit or s2 % unit:
             return False
     return True
 

@@ -25,7 +25,7 @@ import torch.nn as nn
 
 from .. import _ops
 from ..dispatch import ATTENTION_TAIL_ROWS, LAYER_TAIL_SHAPES, LAYERNORM_QKV_WIDTHS, attention_tail_supported
-from .hip_linear import _fp16_linear_ok, _gpu, _norm_ok
+from .hip_linear import _fp16_linear_ok, _fp16_params_ok, _gpu, _norm_ok, _norm_params_ok
 
 
 def layer_tail_supported(d_model: int, ffn_dim: int) -> bool:
@@ -70,6 +70,38 @@ def _q_scale(q_scale: Optional[float]) -> float:
     return q
 
 
+def _tail_tensors(
+    d: int, out_proj: nn.Linear, norm2: nn.LayerNorm, ffn_in: nn.Linear, ffn_out: nn.Linear, next_norm: nn.LayerNorm,
+    next_qkv_proj: Optional[nn.Linear],
+):
+    """The layer tail's parameters, each looked up once (nn.Module attribute lookups are most of
+    such a call's host time): ``(tensors, qkv weight, qkv bias)``, or None where they do not fit."""
+    w_o, b_o = out_proj.weight, out_proj.bias
+    w_in, b_in = ffn_in.weight, ffn_in.bias
+    w_out, b_out = ffn_out.weight, ffn_out.bias
+    ln2_w, ln2_b = norm2.weight, norm2.bias
+    next_w, next_b = next_norm.weight, next_norm.bias
+    w_qkv = b_qkv = None
+    if next_qkv_proj is not None:
+        w_qkv, b_qkv = next_qkv_proj.weight, next_qkv_proj.bias
+        if not (_fp16_params_ok(w_qkv, b_qkv) and next_qkv_proj.in_features == d
+                and next_qkv_proj.out_features == 3 * d):
+            return None
+    if not (
+        out_proj.in_features == out_proj.out_features == d
+        and ffn_in.in_features == d
+        and ffn_out.in_features == ffn_in.out_features
+        and ffn_out.out_features == d
+        and _fp16_params_ok(w_o, b_o)
+        and _fp16_params_ok(w_in, b_in)
+        and _fp16_params_ok(w_out, b_out)
+        and _norm_params_ok(norm2, ln2_w, ln2_b, d)
+        and _norm_params_ok(next_norm, next_w, next_b, d)
+    ):
+        return None
+    return [w_o, b_o, ln2_w, ln2_b, w_in, b_in, w_out, b_out, next_w, next_b], w_qkv, b_qkv
+
+
 def fused_layer_tail(
     ctx: torch.Tensor,
     residual: torch.Tensor,
@@ -91,31 +123,21 @@ def fused_layer_tail(
     (ignored for the last layer, which has no next QKV).
     """
     d = ctx.shape[-1] if ctx.dim() else 0
-    f = ffn_in.out_features
-    last = next_qkv_proj is None
+    params = _tail_tensors(d, out_proj, norm2, ffn_in, ffn_out, next_norm, next_qkv_proj)
     if not (
         _gpu(ctx)
         and ctx.dtype == torch.float16
         and _gpu(residual)
         and residual.dtype == torch.float32
         and residual.shape == ctx.shape
-        and out_proj.in_features == out_proj.out_features == d
-        and ffn_in.in_features == d
-        and ffn_out.in_features == f
-        and ffn_out.out_features == d
-        and all(_fp16_linear_ok(m) for m in (out_proj, ffn_in, ffn_out))
-        and _norm_ok(norm2, d)
-        and _norm_ok(next_norm, d)
-        and (last or (_fp16_linear_ok(next_qkv_proj) and next_qkv_proj.in_features == d
-                      and next_qkv_proj.out_features == 3 * d))
-        and layer_tail_supported(d, f)
+        and params is not None
+        and layer_tail_supported(d, ffn_in.out_features)
     ):
         raise ValueError("unsupported fused layer-tail inputs")
-    tensors = [out_proj.weight, out_proj.bias, norm2.weight, norm2.bias, ffn_in.weight, ffn_in.bias,
-               ffn_out.weight, ffn_out.bias, next_norm.weight, next_norm.bias]
+    tensors, w_qkv, b_qkv = params
     return _ops.layer_tail(
-        ctx, residual, tensors, None if last else next_qkv_proj.weight, None if last else next_qkv_proj.bias,
-        float(norm2.eps), float(next_norm.eps), int(variant), 0.0 if last else _q_scale(q_scale),
+        ctx, residual, tensors, w_qkv, b_qkv, float(norm2.eps), float(next_norm.eps), int(variant),
+        0.0 if next_qkv_proj is None else _q_scale(q_scale),
     )
 
 
@@ -147,32 +169,22 @@ def fused_attention_layer_tail(
     ``fused_layer_tail``.  Returns ``(residual_out, next qkv)``, or ``(residual_out,
     next_norm(residual_out))`` in FP32 when ``next_qkv_proj`` is None (last layer).
     """
-    ok = _gpu(qkv) and qkv.dtype == torch.float16 and qkv.dim() == 3 and qkv.is_contiguous()
     d = residual.shape[-1] if residual.dim() else 0
-    f = ffn_in.out_features
-    last = next_qkv_proj is None
+    params = _tail_tensors(d, out_proj, norm2, ffn_in, ffn_out, next_norm, next_qkv_proj)
     if not (
-        ok
+        _gpu(qkv)
+        and qkv.dtype == torch.float16
+        and qkv.dim() == 3
         and _gpu(residual)
         and residual.dtype == torch.float32
         and residual.dim() == 3
-        and residual.is_contiguous()
         and qkv.shape == (*residual.shape[:-1], 3 * d)
-        and out_proj.in_features == out_proj.out_features == d
-        and ffn_in.in_features == d
-        and ffn_out.in_features == f
-        and ffn_out.out_features == d
-        and all(_fp16_linear_ok(m) for m in (out_proj, ffn_in, ffn_out))
-        and _norm_ok(norm2, d)
-        and _norm_ok(next_norm, d)
-        and (last or (_fp16_linear_ok(next_qkv_proj) and next_qkv_proj.in_features == d
-                      and next_qkv_proj.out_features == 3 * d))
-        and attention_layer_tail_supported(d, f, heads, residual.shape[1])
+        and params is not None
+        and attention_layer_tail_supported(d, ffn_in.out_features, heads, residual.shape[1])
     ):
         raise ValueError("unsupported fused attention layer-tail inputs")
-    tensors = [out_proj.weight, out_proj.bias, norm2.weight, norm2.bias, ffn_in.weight, ffn_in.bias,
-               ffn_out.weight, ffn_out.bias, next_norm.weight, next_norm.bias]
+    tensors, w_qkv, b_qkv = params
     return _ops.attention_layer_tail(
-        qkv, residual, tensors, None if last else next_qkv_proj.weight, None if last else next_qkv_proj.bias,
-        int(heads), float(scale), bool(causal), float(norm2.eps), float(next_norm.eps),
+        qkv, residual, tensors, w_qkv, b_qkv, int(heads), float(scale), bool(causal), float(norm2.eps),
+        float(next_norm.eps),
     )

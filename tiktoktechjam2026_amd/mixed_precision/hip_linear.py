@@ -37,27 +37,37 @@ def _gpu(t: torch.Tensor) -> bool:
     return t.is_cuda and t.is_contiguous()
 
 
-def _fp16_linear_ok(linear: nn.Linear) -> bool:
+def _fp16_params_ok(weight: torch.Tensor, bias: Optional[torch.Tensor]) -> bool:
     return (
-        linear.weight.is_cuda
-        and linear.weight.dtype == torch.float16
-        and linear.weight.is_contiguous()
-        and linear.bias is not None
-        and linear.bias.dtype == torch.float16
-        and linear.bias.is_contiguous()
+        weight.is_cuda
+        and weight.dtype == torch.float16
+        and weight.is_contiguous()
+        and bias is not None
+        and bias.dtype == torch.float16
+        and bias.is_contiguous()
     )
 
 
+def _fp16_linear_ok(linear: nn.Linear) -> bool:
+    return _fp16_params_ok(linear.weight, linear.bias)
+
+
 def _norm_ok(norm: nn.LayerNorm, width: int) -> bool:
+    return _norm_params_ok(norm, norm.weight, norm.bias, width)
+
+
+def _norm_params_ok(
+    norm: nn.LayerNorm, weight: Optional[torch.Tensor], bias: Optional[torch.Tensor], width: int
+) -> bool:
     return (
         tuple(norm.normalized_shape) == (width,)
-        and norm.weight is not None
-        and norm.bias is not None
-        and norm.weight.is_cuda
-        and norm.weight.dtype == torch.float32
-        and norm.bias.dtype == torch.float32
-        and norm.weight.is_contiguous()
-        and norm.bias.is_contiguous()
+        and weight is not None
+        and bias is not None
+        and weight.is_cuda
+        and weight.dtype == torch.float32
+        and bias.dtype == torch.float32
+        and weight.is_contiguous()
+        and bias.is_contiguous()
     )
 
 
@@ -76,17 +86,18 @@ def mixed_linear(
     variant: int = 0,
 ) -> torch.Tensor:
     """``act(fp16(x) @ W^T + b)`` with FP32 accumulation; act = exact GELU if ``fuse_gelu``."""
+    weight, bias = linear.weight, linear.bias
     if not (
         _gpu(x)
         and x.dtype in (torch.float16, torch.float32)
-        and _fp16_linear_ok(linear)
+        and _fp16_params_ok(weight, bias)
         and output_dtype in (torch.float16, torch.float32)
         and x.shape[-1] == linear.in_features
         and linear.in_features % 8 == 0
         and linear.out_features % 8 == 0
     ):
         raise ValueError("unsupported mixed projection inputs")
-    return _ops.linear(x, linear.weight, linear.bias, _code(output_dtype), bool(fuse_gelu), int(variant))
+    return _ops.linear(x, weight, bias, _code(output_dtype), bool(fuse_gelu), int(variant))
 
 
 def mixed_linear_q_scaled(

@@ -280,7 +280,8 @@ class MixedPrecisionTransformer(nn.Module):
             effective_mask = effective_mask.contiguous()
         causal = bool(self.config.causal)
         stream_dtype = self.route.normalized_dtype
-        n_layers = len(self.layers)
+        layers = list(self.layers)
+        n_layers = len(layers)
 
         if self.route.fuse_layer_tail:
             normalized = self._forward_layer_tail(x, effective_mask, causal)
@@ -288,13 +289,13 @@ class MixedPrecisionTransformer(nn.Module):
                 return normalized.masked_fill(~effective_mask[..., None], 0)
             return normalized
 
-        normalized = layer_norm(x, self.layers[0].norm1, normalized_dtype=stream_dtype)
-        for index, layer in enumerate(self.layers):
+        normalized = layer_norm(x, layers[0].norm1, normalized_dtype=stream_dtype)
+        for index, layer in enumerate(layers):
             x, normalized_ffn = layer.attention(
                 normalized, effective_mask, causal, residual_fp32=x, next_norm=layer.norm2
             )
             last = index + 1 == n_layers
-            next_norm = self.final_norm if last else self.layers[index + 1].norm1
+            next_norm = self.final_norm if last else layers[index + 1].norm1
             x, normalized = layer.ffn(
                 normalized_ffn, x, next_norm, torch.float32 if last else stream_dtype, out=out if last else None,
                 last=last,
@@ -309,7 +310,7 @@ class MixedPrecisionTransformer(nn.Module):
 
 def _forward_layer_tail_impl(model: "MixedPrecisionTransformer", x, key_valid, causal):
     route = model.route
-    layers = model.layers
+    layers = list(model.layers)
     if dispatch.attention_tail_for(route, x.shape[1], key_valid is not None):
         # 1 + L launches: each layer's attention runs inside its layer-tail kernel
         qkv = layer_norm_qkv(x, layers[0].norm1, layers[0].attention.qkv_proj, variant=route.head_variant)
