@@ -398,6 +398,12 @@ def test_ffn_wide_residual_layernorm(hip_device, f, m, variant):
     _check_ffn(hip_device, 256, f, m, variant, torch.float16)
 
 
+@pytest.mark.parametrize("d,f,m", [(256, 64, 9), (256, 1024, 16384), (256, 1024, 16385), (512, 192, 1), (512, 2048, 25000)])
+def test_ffn_built_in_choice(hip_device, d, f, m):
+    """Variant 0 at d_model 256 (up to 16,384 rows) and 512: separate projections and LayerNorm."""
+    _check_ffn(hip_device, d, f, m, 0, torch.float16)
+
+
 def test_ffn_wide_fp32_input(hip_device):
     _check_ffn(hip_device, 256, 1024, 777, 4, torch.float32)
 

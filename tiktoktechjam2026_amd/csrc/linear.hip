@@ -1635,6 +1635,24 @@ extern "C" int mpk_linear_qscaled(const void* x, int x_dtype, const void* w, con
   return (int)e;
 }
 
+// Row counts for which projection + residual + LayerNorm at N = 256 / 512 runs as the ring
+// projection (residual in its epilogue, R' into residual_out) and a LayerNorm launch over R'.
+// The fused tiles hold whole rows: few rows leave most CUs idle (128 x 512 tiles: 64 workgroups
+// at 8,192 rows), while the ring tiles shrink with the call.  Measured on MI355X with K = N,
+// us, fused -> two launches: N 512: 16 rows 23.8 -> 8.6, 4,096 39.5 -> 16.2, 16,384 42.8 -> 29.1,
+// 24,576 42.8 -> 41.4, 32,768 48.3 -> 51.8; N 256: 16 rows 6.9 -> 8.7, 64 9.6 -> 7.3, 4,096
+// 14.8 -> 9.7, 16,384 18.8 -> 16.7, 32,768 21.0 -> 26.2.
+static bool ln_split_applies(bool f16_in, int64_t m, int n, int k) {
+  return f16_in && k % 64 == 0 && (n == 512 ? m <= 24576 : n == 256 && m > 32 && m <= 16384);
+}
+
+static int linear_ln_split(const LinearArgs& a, bool normalized_f32, void* stream) {
+  const int e = mpk_linear_residual(a.x, kF16, a.w, a.bias, a.residual, a.residual_out, a.m, a.n, a.k, 0, stream);
+  if (e != MPK_OK) return e;
+  return mpk_layernorm(a.residual_out, nullptr, a.gamma, a.beta, nullptr, a.y, normalized_f32 ? kF32 : kF16, a.m, a.n,
+                       a.eps, stream);
+}
+
 extern "C" int mpk_linear_residual_layernorm_auto_variant(int64_t m, int32_t d) {
   if (d == 256) return 3;
   return m >= 128 * 512 ? 2 : 1;
@@ -1653,8 +1671,6 @@ extern "C" int mpk_linear_residual_layernorm(const void* x, int x_dtype, const v
       !aligned16(beta) || !aligned16(residual_out) || !aligned16(normalized_out))
     return MPK_EALIGN;
   if (m == 0) return MPK_OK;
-  if (variant == 0) variant = mpk_linear_residual_layernorm_auto_variant(m, d);
-  if (variant < 1 || variant > 4) return MPK_EUNSUPPORTED;
   LinearArgs a{};
   a.x = x; a.w = static_cast<const _Float16*>(w); a.bias = static_cast<const _Float16*>(b); a.y = normalized_out;
   a.residual = residual; a.gamma = gamma; a.beta = beta; a.residual_out = residual_out;
@@ -1662,6 +1678,11 @@ extern "C" int mpk_linear_residual_layernorm(const void* x, int x_dtype, const v
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipError_t e;
   const bool xf = x_dtype == kF32, of = normalized_dtype == kF32;
+  if (variant == 0) {
+    if (ln_split_applies(!xf, m, d, d)) return linear_ln_split(a, of, stream);
+    variant = mpk_linear_residual_layernorm_auto_variant(m, d);
+  }
+  if (variant < 1 || variant > 4) return MPK_EUNSUPPORTED;
   if (xf) e = of ? linear_ln<float, float>(variant, a, s) : linear_ln<float, _Float16>(variant, a, s);
   else e = of ? linear_ln<_Float16, float>(variant, a, s) : linear_ln<_Float16, _Float16>(variant, a, s);
   return (int)e;
@@ -1704,6 +1725,7 @@ extern "C" int mpk_linear_add_layernorm(const void* x, int x_dtype, const void* 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipError_t e;
   const bool xf = x_dtype == kF32, of = normalized_dtype == kF32;
+  if (ln_split_applies(!xf, m, n, k)) return linear_ln_split(a, of, stream);
   // FP16 X with d = K = 256 and fewer 256-row tiles than a device has CUs: the
   // weights-resident whole-row kernel (16-row wave tiles fill the device; measured on MI355X:
   // 22 vs 42 us at 32,771 rows, 18 vs 30 us at 8,192; level at 65,536, the large tiles ahead

@@ -155,6 +155,22 @@ std::tuple<Tensor, Tensor> linear_add_layer_norm(const Tensor& x, const Tensor& 
   return {residual_out, normalized};
 }
 
+// FP16 FFNs at d_model 256 / 512 up to these row counts run as projection + GELU (hidden in a
+// temporary of at most 512 MB from torch's caching allocator), projection + residual, and
+// LayerNorm.  The fused kernels walk the hidden layer in 32-wide chunks on one workgroup per
+// 128 tokens (d 256) or 64 (d 512), so a short call takes as long as a full device of rows.
+// Measured on MI355X, us, fused -> separate: d 256, F 1024: 16 rows
+// 42.8 -> 11.9, 4,096 50.9 -> 19.8, 16,384 52.6 -> 44.3, 32,768 59.6 -> 74.7; F 256: 4,096
+// 24.6 -> 13.6, 16,384 26.7 -> 24.4, 32,768 29.6 -> 42.6; d 512, F 2048: slower fused at every
+// row count (32,768: 848 -> 214).
+constexpr int64_t kSplitFfnRows256 = 16384;
+constexpr int64_t kSplitFfnHidden = int64_t{1} << 28;  // elements
+
+bool split_ffn(const Tensor& x, int64_t d, int64_t f, int64_t variant) {
+  return variant == 0 && x.scalar_type() == at::kHalf && f % 64 == 0 &&
+         rows(x, d) * f <= kSplitFfnHidden && (d == 512 || (d == 256 && rows(x, d) <= kSplitFfnRows256));
+}
+
 // residual_out undefined: only `normalized` is stored
 void launch_ffn(const Tensor& x, const Tensor& w_in, const Tensor& b_in, const Tensor& w_out, const Tensor& b_out,
                 const Tensor& residual, const Tensor& gamma, const Tensor& beta, double eps, int64_t variant,
@@ -162,6 +178,21 @@ void launch_ffn(const Tensor& x, const Tensor& w_in, const Tensor& b_in, const T
   const int64_t f = w_in.size(0), d = w_in.size(1);
   require_aligned("unsupported fused FFN inputs", x, w_in, b_in, w_out, b_out, residual, gamma, beta, normalized);
   if (residual_out.defined()) require_aligned("unsupported fused FFN inputs", residual_out);
+  if (split_ffn(x, d, f, variant)) {
+    const int64_t m = rows(x, d);
+    const Tensor hidden = at::empty({m, f}, x.options());
+    const Tensor r = residual_out.defined() ? residual_out : at::empty_like(residual);
+    check(mpk_linear(x.data_ptr(), MPK_F16, w_in.data_ptr(), b_in.data_ptr(), hidden.data_ptr(), MPK_F16, 1, m,
+                     (int32_t)f, (int32_t)d, 0, stream(x)),
+          "mpk_linear");
+    check(mpk_linear_residual(hidden.data_ptr(), MPK_F16, w_out.data_ptr(), b_out.data_ptr(), f32(residual),
+                              f32_out(r), m, (int32_t)d, (int32_t)f, 0, stream(x)),
+          "mpk_linear_residual");
+    check(mpk_layernorm(f32(r), nullptr, f32(gamma), f32(beta), nullptr, normalized.data_ptr(),
+                        dtype_code(normalized), m, (int32_t)d, (float)eps, stream(x)),
+          "mpk_layernorm");
+    return;
+  }
   check(mpk_ffn_residual_layernorm(x.data_ptr(), dtype_code(x), w_in.data_ptr(), b_in.data_ptr(), w_out.data_ptr(),
                                    b_out.data_ptr(), f32(residual), f32(gamma), f32(beta),
                                    residual_out.defined() ? f32_out(residual_out) : nullptr, normalized.data_ptr(),
