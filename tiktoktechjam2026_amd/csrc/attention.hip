@@ -70,28 +70,53 @@ __device__ __forceinline__ h8 buffer_load8_scaled(__amdgpu_buffer_rsrc_t r, uint
   return h;
 }
 
-// Largest |x| over rows [0, rows) x cols (cols % 8 == 0) of an FP32 matrix, reduced over
-// the workgroup (NT threads; red: NT / 64 floats of LDS).  Every thread must call it.
+// Largest |x| over rows [0, rows) x cols (cols % 8 == 0) of the FP32 matrices k and v, reduced
+// over the workgroup (NT threads; red: 2 NT / 64 floats of LDS).  Every thread must call it.
+// Both matrices together, four chunks of each in flight: with one chunk at a time the pass was a
+// chain of rows * cols / 8 / NT memory latencies per matrix and took most of a short call
+// (B16 H4 S1024 hd 32, MI355X: 27.3 -> 24.0 us; B1 H8 S3805 hd 64 with a padded tail 147 -> 69).
 template <int NT>
-__device__ float wg_absmax(const float* base, int64_t row_stride, int rows, int cols, float* red) {
-  float m = 0.f;
-  const int cpr = cols / 8;
-  for (int c = threadIdx.x; c < rows * cpr; c += NT) {
-    const float* p = base + (int64_t)(c / cpr) * row_stride + (c % cpr) * 8;
-    const float4 x0 = *reinterpret_cast<const float4*>(p);
-    const float4 x1 = *reinterpret_cast<const float4*>(p + 4);
-    m = fmaxf(m, fmaxf(fmaxf(fabsf(x0.x), fabsf(x0.y)), fmaxf(fabsf(x0.z), fabsf(x0.w))));
-    m = fmaxf(m, fmaxf(fmaxf(fabsf(x1.x), fabsf(x1.y)), fmaxf(fabsf(x1.z), fabsf(x1.w))));
+__device__ void wg_absmax_kv(const float* k, int64_t k_stride, const float* v, int64_t v_stride, int rows, int cols,
+                             float* red, float& k_max, float& v_max) {
+  constexpr int U = 4;
+  const int cpr = cols / 8, n = rows * cpr;
+  float mk = 0.f, mv = 0.f;
+  for (int c0 = threadIdx.x; c0 < n; c0 += U * NT) {
+    float4 x[U][4];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int c = min(c0 + u * NT, n - 1);  // past the end: the last chunk again
+      const int row = c / cpr, col = (c % cpr) * 8;
+      const float* pk = k + (int64_t)row * k_stride + col;
+      const float* pv = v + (int64_t)row * v_stride + col;
+      x[u][0] = *reinterpret_cast<const float4*>(pk);
+      x[u][1] = *reinterpret_cast<const float4*>(pk + 4);
+      x[u][2] = *reinterpret_cast<const float4*>(pv);
+      x[u][3] = *reinterpret_cast<const float4*>(pv + 4);
+    }
+    auto amax = [](const float4& q) { return fmaxf(fmaxf(fabsf(q.x), fabsf(q.y)), fmaxf(fabsf(q.z), fabsf(q.w))); };
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      mk = fmaxf(mk, fmaxf(amax(x[u][0]), amax(x[u][1])));
+      mv = fmaxf(mv, fmaxf(amax(x[u][2]), amax(x[u][3])));
+    }
   }
 #pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  for (int o = 32; o >= 1; o >>= 1) {
+    mk = fmaxf(mk, __shfl_xor(mk, o));
+    mv = fmaxf(mv, __shfl_xor(mv, o));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[threadIdx.x >> 6] = mk;
+    red[NT / 64 + (threadIdx.x >> 6)] = mv;
+  }
   __syncthreads();
-  float r = red[0];
+  k_max = red[0], v_max = red[NT / 64];
 #pragma unroll
-  for (int w = 1; w < NT / 64; ++w) r = fmaxf(r, red[w]);
-  __syncthreads();  // red is reused by the next call
-  return r;
+  for (int w = 1; w < NT / 64; ++w) {
+    k_max = fmaxf(k_max, red[w]);
+    v_max = fmaxf(v_max, red[NT / 64 + w]);
+  }
 }
 
 // Valid-key range of a mask row, for keys [0, kv_end): first_bad = the first key that may not be
@@ -106,10 +131,18 @@ __device__ void mask_range(const uint8_t* valid, int kv_end, int* range, int& fi
   if (threadIdx.x == 0) range[0] = kv_end, range[1] = 0;
   __syncthreads();
   int fb = kv_end, lk = 0;
-  for (int k0 = 64 * wave_id(); k0 < kv_end; k0 += 64 * NW) {
-    const uint64_t ok = __builtin_amdgcn_ballot_w64(k0 + l < kv_end && valid[min(k0 + l, kv_end - 1)] != 0);
-    if (~ok) fb = min(fb, k0 + (int)__builtin_ctzll(~ok));
-    if (ok) lk = k0 + 64 - (int)__builtin_clzll(ok);
+  constexpr int U = 4;  // loads in flight
+  for (int base = 64 * U * wave_id(); base < kv_end; base += 64 * U * NW) {
+    uint8_t byte[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) byte[u] = valid[min(base + 64 * u + l, kv_end - 1)];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k0 = base + 64 * u;
+      const uint64_t ok = __builtin_amdgcn_ballot_w64(k0 + l < kv_end && byte[u] != 0);
+      if (~ok) fb = min(fb, k0 + (int)__builtin_ctzll(~ok));
+      if (ok) lk = k0 + 64 - (int)__builtin_clzll(ok);
+    }
   }
   if (l == 0) {
     atomicMin(&range[0], fb);
@@ -210,11 +243,12 @@ __global__ __launch_bounds__(64 * NW) void attention_kernel(AttnArgs a) {
   constexpr bool F32IN = std::is_same<IT, float>::value;
   int kexp = 0, vexp = 0;
   if constexpr (F32IN) {
-    __shared__ float red[NW];
-    kexp = __builtin_amdgcn_readfirstlane(
-        f32_scale_exp(wg_absmax<NT>(reinterpret_cast<const float*>(Kp), a.ks[2], kv_end, HD, red)));
-    vexp = __builtin_amdgcn_readfirstlane(
-        f32_scale_exp(wg_absmax<NT>(reinterpret_cast<const float*>(Vp), a.vs[2], kv_end, HD, red)));
+    __shared__ float red[2 * NW];
+    float kmax, vmax;
+    wg_absmax_kv<NT>(reinterpret_cast<const float*>(Kp), a.ks[2], reinterpret_cast<const float*>(Vp), a.vs[2], kv_end,
+                     HD, red, kmax, vmax);
+    kexp = __builtin_amdgcn_readfirstlane(f32_scale_exp(kmax));
+    vexp = __builtin_amdgcn_readfirstlane(f32_scale_exp(vmax));
   }
 
   // ---- Q fragments (B operand of S^T = K Q^T), kept in registers ----
@@ -756,11 +790,12 @@ void attention32_kernel(AttnArgs a) {
   constexpr bool F32IN = std::is_same<IT, float>::value;
   int kexp = 0, vexp = 0;
   if constexpr (F32IN) {
-    __shared__ float red[NW];
-    kexp = __builtin_amdgcn_readfirstlane(
-        f32_scale_exp(wg_absmax<NT>(reinterpret_cast<const float*>(Kp), a.ks[2], kv_end, HD, red)));
-    vexp = __builtin_amdgcn_readfirstlane(
-        f32_scale_exp(wg_absmax<NT>(reinterpret_cast<const float*>(Vp), a.vs[2], kv_end, HD, red)));
+    __shared__ float red[2 * NW];
+    float kmax, vmax;
+    wg_absmax_kv<NT>(reinterpret_cast<const float*>(Kp), a.ks[2], reinterpret_cast<const float*>(Vp), a.vs[2], kv_end,
+                     HD, red, kmax, vmax);
+    kexp = __builtin_amdgcn_readfirstlane(f32_scale_exp(kmax));
+    vexp = __builtin_amdgcn_readfirstlane(f32_scale_exp(vmax));
   }
 
   // Q fragments (B operand of S^T): query q, head dims 16 st + 8 hf .. +7; negated for a

@@ -212,8 +212,9 @@ __device__ __forceinline__ void pin_f32x8(float* x) {
 // where the erf formula used before (Abramowitz & Stegun 7.1.26) took a reciprocal, an exp2 and
 // 11 others: 48 instead of 60 VALU cycles per wave and element.  Against float64 over [-12, 12]
 // (FP32 emulation of these steps): largest error 2.6e-7 and rms 4.5e-8, before 3.3e-7 and
-// 7.6e-8; relative error in [-5.5, -0.5] 3.1e-4, before 2.5e-3.  MI355X, variant 9 / 8: 32,768 x
-// 2048 x 512 92.4 -> 86.0 us, 65,536 x 1024 x 256 60.6 -> 57.4, 32,768 x 4096 x 1024 302 -> 294.
+// 7.6e-8; relative error in [-5.5, -0.5] 3.1e-4, before 2.5e-3.  Projections with it
+// on MI355X, us, before -> after: 32,768 x 2048 x 512 92.4 -> 86.0, 65,536 x 1024 x 256 60.6 -> 57.4,
+// 32,768 x 4096 x 1024 302 -> 294.
 __device__ __forceinline__ float gelu_erf(float x) {
   constexpr float c1 = -1.151126742362976f, c2 = -0.4590495526790619f, c3 = -0.05292149633169174f;
   constexpr float c4 = 0.0076178559102118015f, c5 = -0.0005247833323664963f, c6 = -3.8311085518216714e-05f;
