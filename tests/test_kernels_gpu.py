@@ -1070,3 +1070,16 @@ def test_attention_prescaled_rejects(hip_device):
     _, q, k, v = _packed_qkv(1, 64, 2, 32, 5, hip_device, torch.float32)
     with pytest.raises(ValueError):
         attention_prescaled(q, k, v)
+
+
+def test_raw_operator_dimensions(hip_device):
+    """The operators below the checking wrappers: attention views without four dimensions are
+    refused, and a 0-d projection input gives the empty-row output shape."""
+    from tiktoktechjam2026_amd import _lib, _ops
+
+    x = _randn((2, 8, 32), 6).to(hip_device, torch.float16)
+    with pytest.raises(ValueError):
+        _ops.attention(x, x, x, None, 1.0, True, _lib.F16, 0)
+    lin = _linear(64, 32, hip_device, 7)
+    y = _ops.linear(x[0, 0, 0].clone(), lin.weight, lin.bias, _lib.F16, False, 0)
+    assert y.shape == (32,)

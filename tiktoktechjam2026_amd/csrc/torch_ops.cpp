@@ -53,6 +53,7 @@ int64_t rows(const Tensor& t, int64_t width) { return width ? t.numel() / width 
 // a contiguous output of t's shape with the last dimension replaced by `width`
 Tensor empty_rows(const Tensor& t, int64_t width, at::ScalarType dtype) {
   c10::DimVector sizes(t.sizes().begin(), t.sizes().end());
+  if (sizes.empty()) sizes.resize(1);  // a 0-d tensor has rows of width 1
   sizes.back() = width;
   return at::empty(sizes, t.options().dtype(dtype));
 }
@@ -239,6 +240,8 @@ Tensor attention_out(const Tensor& q, at::ScalarType dtype, int64_t (&strides)[4
 }
 
 void require_aligned_qkv(const Tensor& q, const Tensor& k, const Tensor& v) {
+  TORCH_CHECK_VALUE(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "unsupported custom-attention input: shape=",
+                    q.sizes(), ", dtype=", q.scalar_type(), " (4 dimensions)");
   const uintptr_t bits = reinterpret_cast<uintptr_t>(q.data_ptr()) | reinterpret_cast<uintptr_t>(k.data_ptr()) |
                          reinterpret_cast<uintptr_t>(v.data_ptr());
   TORCH_CHECK_VALUE(bits % 16 == 0, "unsupported custom-attention input: shape=", q.sizes(), ", dtype=",
