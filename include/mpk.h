@@ -58,8 +58,9 @@ int mpk_layernorm(const float* x, const float* update, const float* gamma, const
  * variant 0: the built-in table (mpk_linear_auto_variant); 1-9 pin a tile shape (all give
  * identical results).  8: 256x256 tiles with LDS-DMA operand staging; 9: X-stationary
  * 256-token tiles with W streamed through LDS (FP16 x, k = 128 or 256, n % 64 == 0).  With
- * variant 0, FP16 x and k % 64 == 0, calls for which the table answers 1-4 (and 8 from k = 2048)
- * run the ring kernel on a tile picked from m, n and k, with identical results.
+ * variant 0, FP16 x and k % 64 == 0, calls for which the table answers 1-4 (and 8 from k = 2048,
+ * or from k = 320 where 256x192 tiles need no more rounds of 256 CUs) run the ring kernel on a
+ * tile picked from m, n and k, with identical results.
  * Replaces: mixed_linear (mixed_precision/triton_linear.py:221-269).
  */
 int mpk_linear(const void* x, int x_dtype, const void* w, const void* b, void* y, int y_dtype, int gelu,

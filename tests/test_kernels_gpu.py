@@ -174,7 +174,7 @@ def test_linear_x_stationary_variant_bit_identical(hip_device, m, n, k):
 @pytest.mark.parametrize(
     "m,n,k",
     [(1, 32, 64), (33, 40, 64), (77, 2048, 512), (1000, 200, 128), (52, 1024, 4096), (1600, 1024, 1024),
-     (5673, 520, 192), (8191, 1000, 320), (16640, 1024, 2112)],
+     (5673, 520, 192), (8191, 1000, 320), (16640, 1024, 2112), (7937, 3072, 320), (24001, 376, 512), (4999, 3064, 320)],
 )
 def test_linear_ring_tiles_bit_identical(hip_device, m, n, k):
     """The built-in choice at K % 64 == 0 (ring kernel: tiles from 32 x 32 to 256 x 256, one to

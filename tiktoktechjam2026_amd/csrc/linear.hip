@@ -1044,11 +1044,15 @@ static hipError_t launch_ring_tile(const LinearArgs& a, hipStream_t s) {
 // copies, last stores).  step / end / start in units of 10 ns, fitted to sweeps on MI355X
 // over 22 shapes from 3 x 2048 x 1536 to 32768 x 2048 x 512 (the tile it picks was within
 // 15 % of the fastest on each): a 128 x 128 tile alone takes 0.5 us per 64 k values, a
-// 32 x 32 one 0.1 us, and the ends cost 0.7-1.7 us of stores and epilogue per tile.
+// 32 x 32 one 0.1 us, and the ends cost 0.7-1.7 us of stores and epilogue per tile.  The two large
+// tiles (1.33 and 1.06 us per 64 k values, ends of 10 us with one workgroup per CU) serve calls
+// that they fill in a round or two: 5000 x 3072 x 1024 39.2 -> 35.7 us (256 x 256), 3000 x 3072 x 1024
+// 32.3 -> 27.2, 2500 x 4096 x 1024 GELU 35.3 -> 29.9, 65536 x 384 x 512 38.0 -> 35.0 (256 x 192).
 struct RingTile {
   int bm, bn, step, end, start;
 };
 constexpr RingTile kRingTiles[] = {
+    {256, 256, 133, 1050, 200}, {256, 192, 106, 1030, 150},
     {128, 128, 50, 170, 550}, {128, 64, 27, 130, 400}, {64, 64, 15, 100, 330}, {32, 64, 10, 75, 270}, {32, 32, 10, 70, 250},
 };
 
@@ -1069,19 +1073,30 @@ static int ring_tile(int64_t m, int n, int k) {
 // K >= 2048.  There the 256 x 256 ring tile's 64-wide chunks win what its missing overlap of
 // tile ends loses: 32768 x 512 x 2048 with residual 81.5 vs 84 us, 8192^3 932 vs 1206 us; at
 // K = 1024 variant 8 is ahead, 310 vs 321 us for 32768 x 4096 with GELU.
-constexpr int kRing256MinK = 2048;
-static bool ring_applies(int variant, int k) {
-  return k % 64 == 0 && k <= (1 << 20) && (variant <= 4 || (variant == 8 && k >= kRing256MinK));
+// Variant 8 also gives way to 256 x 192 ring tiles from K = 320 where they need no more rounds of
+// 256 CUs than its 256 x 256 tiles: as many tiles per CU, each 3/4 of the work (us, 256 x 256 ->
+// 256 x 192: 8192 x 3072 x 1024, 384 / 512 tiles, 62.7 -> 55.3; 8192 x 3072 x 2048 residual 130 -> 110;
+// 16384 x 1536 x 512 36.2 -> 33.0; 40000 x 512 x 2048 residual 140 -> 126).  With a round more they
+// lose (32768 x 1536 x 512 59.0 -> 63.5, 16384 x 3072 x 1024 95.7 -> 105), and at K = 256 the end of a
+// tile outweighs its product (8192 x 3072 x 256 25.1 -> 26.6, 32768 x 768 x 256 24.6 -> 23.4).
+constexpr int kRing256MinK = 2048, kRing192MinK = 320;
+static bool ring_192(int64_t m, int n) {
+  const int64_t rows = (m + 255) / 256;
+  return (rows * ((n + 191) / 192) + 255) / 256 <= (rows * ((n + 255) / 256) + 255) / 256;
+}
+static bool ring_applies(int variant, int64_t m, int n, int k) {
+  return k % 64 == 0 && k <= (1 << 20) && (variant <= 4 || (variant == 8 && (k >= kRing256MinK || (k >= kRing192MinK && ring_192(m, n)))));
 }
 
 template <int EPI, typename OT>
 static hipError_t launch_ring(int variant, const LinearArgs& a, hipStream_t s) {
-  if (variant == 8) return launch_ring_tile<256, 256, 2, 4, 2, EPI, OT>(a, s);
-  switch (ring_tile(a.m, a.n, a.k)) {
-    case 0: return launch_ring_tile<128, 128, 2, 2, 2, EPI, OT>(a, s);
-    case 1: return launch_ring_tile<128, 64, 2, 2, 3, EPI, OT>(a, s);
-    case 2: return launch_ring_tile<64, 64, 2, 2, 5, EPI, OT>(a, s);
-    case 3: return launch_ring_tile<32, 64, 2, 2, 6, EPI, OT>(a, s);
+  switch (variant == 8 ? (ring_192(a.m, a.n) ? 1 : 0) : ring_tile(a.m, a.n, a.k)) {
+    case 0: return launch_ring_tile<256, 256, 2, 4, 2, EPI, OT>(a, s);
+    case 1: return launch_ring_tile<256, 192, 4, 2, 2, EPI, OT>(a, s);
+    case 2: return launch_ring_tile<128, 128, 2, 2, 2, EPI, OT>(a, s);
+    case 3: return launch_ring_tile<128, 64, 2, 2, 3, EPI, OT>(a, s);
+    case 4: return launch_ring_tile<64, 64, 2, 2, 5, EPI, OT>(a, s);
+    case 5: return launch_ring_tile<32, 64, 2, 2, 6, EPI, OT>(a, s);
     default: return launch_ring_tile<32, 32, 2, 1, 10, EPI, OT>(a, s);
   }
 }
@@ -1515,7 +1530,7 @@ static hipError_t linear_variant(int variant, const LinearArgs& a, hipStream_t s
   if (variant == 0) {  // the built-in choice
     variant = mpk_linear_auto_variant(a.m, a.n, a.k);
     if constexpr (std::is_same<XT, _Float16>::value) {
-      if (ring_applies(variant, a.k)) return launch_ring<EPI, OT>(variant, a, s);
+      if (ring_applies(variant, a.m, a.n, a.k)) return launch_ring<EPI, OT>(variant, a, s);
     }
   }
   switch (variant) {
