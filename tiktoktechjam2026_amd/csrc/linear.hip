@@ -1042,8 +1042,9 @@ static hipError_t launch_ring_tile(const LinearArgs& a, hipStream_t s) {
 // Tiles of the ring kernel, and the model that picks one: a CU works through
 // ceil(tiles / 256) tiles of (K / 64) * step + end each, after a fixed start (launch, first
 // copies, last stores).  step / end / start in units of 10 ns, fitted to sweeps on MI355X
-// over 22 shapes from 3 x 2048 x 1536 to 32768 x 2048 x 512 (the tile it picks was within
-// 15 % of the fastest on each): a 128 x 128 tile alone takes 0.5 us per 64 k values, a
+// over 22 shapes from 3 x 2048 x 1536 to 32768 x 2048 x 512 (over 72 other drawn shapes the tile it
+// picks was 4 % slower than the fastest on average; worst 33000 x 192 x 1024, 36.7 vs 24.6 us on
+// 256 x 192): a 128 x 128 tile alone takes 0.5 us per 64 k values, a
 // 32 x 32 one 0.1 us, and the ends cost 0.7-1.7 us of stores and epilogue per tile.  The two large
 // tiles (1.33 and 1.06 us per 64 k values, ends of 10 us with one workgroup per CU) serve calls
 // that they fill in a round or two: 5000 x 3072 x 1024 39.2 -> 35.7 us (256 x 256), 3000 x 3072 x 1024
